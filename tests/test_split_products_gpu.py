@@ -120,6 +120,28 @@ def test_rows_near_the_bottom_of_the_exponent_range(hip, m, k, n, small, large):
     check(hip, b.t(), a.t())
 
 
+@pytest.mark.parametrize("exponent", [-109, -112, -118, -120, -126, -130, -135, -140, -148])
+@pytest.mark.parametrize("m, k, n", [(64, 32, 64), (130, 70, 66), (96, 1000, 640), (2048, 64, 2048), (4096, 40, 4096)])
+def test_rows_that_mix_magnitudes(hip, m, k, n, exponent):
+    """Rows of one and of a number near the bottom of the exponent range, whose
+    partners are zero and large: the planes drop the small number's low bits,
+    and only its product reaches the output. Within the contract's 1e-5 sum
+    |a b|, as left and as right operand."""
+    banner(f"mixed magnitudes {m}x{k}x{n} {exponent}")
+    g = torch.Generator().manual_seed(m + k - exponent)
+    small = (torch.rand(m, generator=g, dtype=torch.float64) + 1) * 2.0 ** exponent
+    a, b = torch.zeros(m, k), torch.zeros(k, n)
+    a[:, 0] = 1.0
+    a[:, k - 3] = small.float()
+    a[m // 2] = 0.0
+    b[k - 3] = 2.0 ** min(-exponent, 120) * (torch.rand(n, generator=g) + 1)
+    b[1, :] = torch.randn(n, generator=g)
+    a, b = a.cuda(), b.cuda()
+    x, y = a.double(), b.double()
+    for got in (product(hip, a, b), product(hip, b.t(), a.t()).t()):
+        assert bool(((got.double() - x @ y).abs() <= 1e-5 * (x.abs() @ y.abs())).all())
+
+
 def test_zeros_are_positive(hip):
     """A product of zeros, signed or not, is +0."""
     banner("zeros")
