@@ -126,7 +126,7 @@ def test_rows_that_mix_magnitudes(hip, m, k, n, exponent):
     """Rows of one and of a number near the bottom of the exponent range, whose
     partners are zero and large: the planes drop the small number's low bits,
     and only its product reaches the output. Within the contract's 1e-5 sum
-    |a b|, as left and as right operand."""
+    |a b| in every orientation, as left and as right operand."""
     banner(f"mixed magnitudes {m}x{k}x{n} {exponent}")
     g = torch.Generator().manual_seed(m + k - exponent)
     small = (torch.rand(m, generator=g, dtype=torch.float64) + 1) * 2.0 ** exponent
@@ -138,8 +138,11 @@ def test_rows_that_mix_magnitudes(hip, m, k, n, exponent):
     b[1, :] = torch.randn(n, generator=g)
     a, b = a.cuda(), b.cuda()
     x, y = a.double(), b.double()
-    for got in (product(hip, a, b), product(hip, b.t(), a.t()).t()):
-        assert bool(((got.double() - x @ y).abs() <= 1e-5 * (x.abs() @ y.abs())).all())
+    bound = 1e-5 * (x.abs() @ y.abs())
+    for left in (a, a.t().contiguous().t()):
+        for right in (b, b.t().contiguous().t()):
+            for got in (product(hip, left, right), product(hip, right.t(), left.t()).t()):
+                assert bool(((got.double() - x @ y).abs() <= bound).all())
 
 
 def test_zeros_are_positive(hip):
