@@ -229,8 +229,9 @@ void launch_split_reduce(const float *partials, int splits, int64_t m, int64_t n
 // products, reduced in a fixed order (deterministic; envelope fidelity like
 // the unsplit kernel).
 // The workspace floats launch_gemm_mfma's chosen split uses for this product:
-// its partials (rows padded to whole quads), or 0 when it runs unsplit.
-int64_t mfma_split_floats(int64_t m, int64_t n, int64_t k, int64_t batches);
+// its partials (rows padded to whole quads), or 0 when it runs unsplit;
+// `ranges`, if given, receives the ranges of k.
+int64_t mfma_split_floats(int64_t m, int64_t n, int64_t k, int64_t batches, int *ranges = nullptr);
 // Whether launch_gemm_mfma takes operands with these strides (else the
 // caller's exact fallback runs). Its products are never -0: every
 // accumulator starts at +0, and a sum of +0 with any zero is +0.

@@ -2262,13 +2262,15 @@ struct topos_hip_program {
     const bool mfma = numerics == TOPOS_HIP_FAST && mfma_serves(ars, acs, brs, bcs, n, k, m);
     int64_t workspace_floats = 0;
     int workspace = -1;
-    if (numerics == TOPOS_HIP_FAST) {
-      workspace_floats = mfma_split_floats(n, m, k, 1);
+    int ranges = 1;
+    if (mfma) {
+      workspace_floats = mfma_split_floats(n, m, k, 1, &ranges);
       if (workspace_floats > 0) workspace = arena_storage(workspace_floats * 4);
     }
     std::ostringstream what;
     what << "gemm " << (numerics == TOPOS_HIP_FAST ? "mfma" : "exact") << " 1x(" << n << "," << m << "," << k
          << ") a[" << ars << "," << acs << "] b[" << brs << "," << bcs << "] transposed";
+    if (ranges > 1) what << " in " << ranges << " ranges";
     std::vector<int> writes = {out};
     if (workspace >= 0) writes.push_back(workspace);
     const int numerics_ = numerics;
@@ -2376,13 +2378,15 @@ struct topos_hip_program {
     // Scratch for the partial products of a split along k (fast posture).
     int64_t workspace_floats = 0;
     int workspace = -1;
-    if (numerics == TOPOS_HIP_FAST) {
-      workspace_floats = mfma_split_floats(m, n, k, batch.count);
+    int ranges = 1;
+    if (mfma_product[i]) {
+      workspace_floats = mfma_split_floats(m, n, k, batch.count, &ranges);
       if (workspace_floats > 0) workspace = arena_storage(workspace_floats * 4);
     }
     std::ostringstream what;
     what << "gemm " << (numerics == TOPOS_HIP_FAST ? "mfma" : "exact") << " " << batches << "x(" << m << "," << n
          << "," << k << ") a[" << ars << "," << acs << "] b[" << brs << "," << bcs << "]";
+    if (ranges > 1) what << " in " << ranges << " ranges";
     std::vector<int> writes = {out};
     if (workspace >= 0) writes.push_back(workspace);
     auto bias = std::make_shared<BiasEpilogue>();

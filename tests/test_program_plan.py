@@ -202,6 +202,22 @@ print(p.info["launches"], d.count("gemm mfma"), d.count(": rows ["))
     assert launches > 60 and gemms >= 2 * 3 * 8 and rows >= 5, out
 
 
+def test_large_products_take_no_partials():
+    # Products whose tiles fill the chip run in one range of k: their partials
+    # would be several times the output (16 GiB for the first). Smaller ones
+    # are cut as short as f32 matrix-core kernels cut them.
+    out = run(r'''
+for m, k, c in ((32768, 16384, 32768), (128256, 8192, 4096), (4096, 4096, 4096), (2048, 8192, 2048), (2560, 8192, 2560)):
+    tape = t.Tape()
+    p = DeviceProgram(tape, [tape.input((m, k)).matmul(tape.input((k, c)))], numerics=n.FAST)
+    line, = [l for l in p.describe.splitlines() if "gemm mfma" in l]
+    print(line.split(" in ")[1].split()[0] if " ranges" in line else 1, p.info["arena_bytes"] / (4 * m * c))
+''')
+    rows = [tuple(map(float, line.split())) for line in out.strip().splitlines()]
+    assert all(ranges == 1 and size < 1.01 for ranges, size in rows[:3]), out
+    assert all(2 <= ranges <= 8 and size < ranges + 1.01 for ranges, size in rows[3:]), out
+
+
 def test_consecutive_chains_join():
     # a = x*x + y has two consumers, so it is materialised; the chains that
     # follow over the same shape join its launch (one kernel, several
