@@ -159,6 +159,22 @@ def test_ranges_are_as_short_as_the_f32_kernels(hip, m, k, n, reach):
     assert error <= 1.79e-8 * reach ** 0.5, error
 
 
+@pytest.mark.parametrize("exponent", [0, -118, -126])
+@pytest.mark.parametrize("m, k, n", [(70, 1, 10), (2048, 1, 2048), (2048, 2, 2048), (300, 2, 70), (1030, 3, 1027),
+                                     (8192, 3, 768)])
+def test_products_of_few_terms(hip, m, k, n, exponent):
+    """A chain of k fused multiply-adds rounds k times, each at most 2^-24 of
+    sum |a b| (or half of 2^-149): one term is the correctly rounded product."""
+    banner(f"few terms {m}x{k}x{n} {exponent}")
+    a = operand(41, m, k, False) * 2.0 ** (exponent // 2)
+    b = operand(42, k, n, True) * 2.0 ** (exponent - exponent // 2)
+    x, y = a.double(), b.double()
+    got = product(hip, a, b)
+    if k == 1:
+        assert bool((got == a * b).all())
+    assert bool(((got.double() - x @ y).abs() <= k * (2.0 ** -24 * (x.abs() @ y.abs()) + 2.0 ** -150)).all())
+
+
 def test_zeros_are_positive(hip):
     """A product of zeros, signed or not, is +0."""
     banner("zeros")
