@@ -319,8 +319,7 @@ def test_adamw_steps_match_the_rule(hip):
 def test_split_product_with_odd_width_and_fused_bias(hip):
     """A Linear layer whose product has enough tiles to fill the chip but
     fills its last round poorly, so it splits along k, with a width of 20001
-    (rows that are not whole quads: the partials are reduced in quads of the
-    flat output) and the bias added by that reduction: within the envelope
+    (rows that are not whole quads: the partials' rows are padded to them) and the bias added by that reduction: within the envelope
     |c - exact| <= 1e-5 * sum_k |x_ik w_kj| + 1 ulp for the bias addition."""
     banner("program split product, odd width, fused bias")
     tape = t.Tape()
@@ -334,7 +333,7 @@ def test_split_product_with_odd_width_and_fused_bias(hip):
     bs = g.normal(20001, 1.0)
     want = run_oracle(tape, [y], [ws, bs], {x.node.slot: xs})[y.id].astype(np.float64)
     got, program = run_device(tape, [y], [ws, bs], {x.node.slot: xs}, numerics=hip.FAST)
-    assert "+bias" in program.describe
+    assert "ranges +bias" in program.describe
     bound = 1e-5 * (np.abs(xs.astype(np.float64)) @ np.abs(ws.astype(np.float64)))
     bound += np.spacing(np.abs(want).astype(np.float32)).astype(np.float64)
     assert (np.abs(got[y.id].astype(np.float64) - want) <= bound).all()

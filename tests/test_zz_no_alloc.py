@@ -28,7 +28,7 @@ import oracle  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 # (m, k, n, seed). Under Fast both split k: 16 partials of 512 x 512 (16 MiB)
-# then 8 of 256 x 384, each within the 64 MiB array.
+# then 16 of 256 x 384, each within the 64 MiB array.
 CASES = [(512, 4096, 512, 21), (256, 2048, 384, 22)]
 
 
@@ -94,16 +94,22 @@ def test_noalloc_product_equals_allocating_product(hip, posture, transposed):
 
 
 def test_noalloc_splits_within_its_array(hip):
-    """2048 x 2048 over k = 8192 splits six ways under Fast on the allocating
-    entry (96 MiB of partials); the no-allocation entry takes the four ranges
+    """2560 x 2560 over k = 8192 splits five ways under Fast on the allocating
+    entry (125 MiB of partials); the no-allocation entry takes the two ranges
     its 64 MiB array holds. Both within the envelope (rows sampled against the
     oracle); Exact needs no scratch and stays bitwise equal."""
     import torch
 
+    from poorgrad_amd.program import DeviceProgram
+    from poorgrad_amd.topos import Tape
     from tests.conftest import banner
     from tests.gpu_util import assert_bitwise, to_device
 
-    m, k, n = 2048, 8192, 2048
+    m, k, n = 2560, 8192, 2560
+    tape = Tape()
+    plan = DeviceProgram(tape, [tape.input((m, k)).matmul(tape.input((k, n)))], numerics=hip.FAST).describe
+    ranges = int(plan.split(" in ")[1].split(" ranges")[0])
+    assert 4 * ranges * m * n > 64 << 20 >= 4 * 2 * m * n, plan
     banner(f"noalloc: capped split {m}x{k}x{n}")
     g = oracle.Generator(31)
     a = g.normal(m * k, 1.0).reshape(m, k)
