@@ -1122,6 +1122,15 @@ struct RowLayout {
   std::vector<int> avail, slot, max_slot, total_slot, lns_slot;
   std::vector<RowFold> folds;
   int passes = 0, slots = 0, levels = 0;
+  int folds_per_pass() const {
+    int most = 1;
+    for (int q = 0; q < passes; ++q) {
+      int k = 0;
+      for (const RowFold &f : folds) k += f.pass == q;
+      most = std::max(most, k);
+    }
+    return most;
+  }
 };
 
 RowLayout lay_out(const RowProgram &p) {
@@ -1664,12 +1673,7 @@ Generated generate_row_streaming(const RowProgram &p, const RowLayout &l, const 
   const int PP = G * SV / 256;        // points per lane per slab
   const int per = 256 / G;            // lanes per row in a max fold
   const int n = m.n;
-  int folds_per_pass = 1;
-  for (int q = 0; q < l.passes; ++q) {
-    int k = 0;
-    for (const RowFold &f : l.folds) k += f.pass == q;
-    folds_per_pass = std::max(folds_per_pass, k);
-  }
+  const int folds_per_pass = l.folds_per_pass();
   std::ostringstream s;
   s << preamble();
   s << signature(m.e, m.tail()) << " {\n  topos_tables_init();\n";
@@ -1889,7 +1893,13 @@ Generated generate_row_program(const RowProgram &p) {
   for (int d = 0; d < p.rank; ++d)
     if (p.shape[d] <= 0) throw InvalidArgument{"row program shape"};
   const RowLayout l = lay_out(p);
-  const RowBlocking blocking = row_blocking(p);
+  RowBlocking blocking = row_blocking(p);
+  // A pass keeps a slab of every fold's operand in LDS (160 KB): narrower slabs
+  // where many folds' would not fit, down to one point a lane.
+  const int folds = l.folds_per_pass();
+  auto bytes = [&] { return 4 * (folds * blocking.rows * (blocking.slab + 4) + std::max(l.slots, 1) * blocking.rows); };
+  while (!blocking.resident && bytes() > 163840 - 4096 && blocking.rows * blocking.slab > 256 * blocking.width)
+    blocking.slab /= 2;
   if (blocking.resident) return generate_row_resident(p, l, blocking);
   return generate_row_streaming(p, l, blocking);
 }

@@ -218,6 +218,22 @@ for m, k, c in ((32768, 16384, 32768), (128256, 8192, 4096), (4096, 4096, 4096),
     assert all(2 <= ranges <= 8 and size < ranges + 1.01 for ranges, size in rows[3:]), out
 
 
+def test_a_row_program_of_many_folds_fits():
+    # Nine sums over streamed rows in one pass, each with its slab in LDS:
+    # rows that are whole quads and rows that are not.
+    out = run(r'''
+for columns in (2049, 4096):
+    tape = t.Tape()
+    x = tape.input((40, columns))
+    total = None
+    for i in range(9):
+        s = (x * tape.parameter((columns,)).broadcast_along(0, x)).sum_along(1)
+        total = s if total is None else total + s
+    print(DeviceProgram(tape, [total]).describe)
+''')
+    assert out.count(", 9 folds, ") == 2, out
+
+
 def test_consecutive_chains_join():
     # a = x*x + y has two consumers, so it is materialised; the chains that
     # follow over the same shape join its launch (one kernel, several

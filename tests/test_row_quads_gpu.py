@@ -1,6 +1,6 @@
 """Row programs over rows that are not whole quads (poorgrad_amd/csrc/codegen.cpp,
-row_quads): four columns a point with the row's last quad lane by lane, bit for
-bit against the oracle, on both layouts (resident up to 2048 columns, streamed
+row_quads): four columns a point, the row's last, partial one from the row's last
+four columns or lane by lane, bit for bit against the oracle, on both layouts (resident up to 2048 columns, streamed
 beyond), at any base alignment, with special values in the partial quad, and
 through programs whose inputs are broadcast along or across the row or
 selected by index."""
@@ -78,3 +78,46 @@ def test_odd_row_programs_bit_identical(hip, columns):
     got, _ = run_device(tape, [weights, terms], [], numerics=hip.EXACT, **feeds)
     for root in (weights, terms):
         assert_bitwise(got[root.id], want[root.id], f"root {root.id}")
+
+
+@pytest.mark.parametrize("rows, columns", [(40, 2049), (9000, 2305), (70000, 2051), (40, 4096)])
+def test_many_folds_over_streamed_rows(hip, rows, columns):
+    """Nine row sums in one pass, over slabs narrowed to fit LDS."""
+    from poorgrad_amd.topos import Tape
+
+    banner(f"many folds {rows}x{columns}")
+    g = oracle.Generator(columns)
+    x = g.normal(rows * columns, 1.0).reshape(rows, columns)
+    scales = [g.normal(columns, 1.0) for _ in range(9)]
+    tape = Tape()
+    s = tape.input((rows, columns))
+    total = None
+    for _ in scales:
+        part = (s * tape.parameter((columns,)).broadcast_along(0, s)).sum_along(1)
+        total = part if total is None else total + part
+    got, program = run_device(tape, [total], scales, dense={0: x}, numerics=hip.EXACT)
+    assert " 9 folds, " in program.describe
+    rows_checked = np.unique(np.r_[0:3, rows // 2, rows - 3:rows])
+    want = None
+    for scale in scales:
+        terms = x[rows_checked] * scale
+        part = terms[:, 0].copy()
+        for j in range(1, columns):
+            part = part + terms[:, j]
+        want = part if want is None else want + part
+    assert_bitwise(got[total.id][rows_checked], want, f"many folds {rows}x{columns}")
+
+
+@pytest.mark.parametrize("rows, columns", [(1343, 50021), (262147, 257), (22370, 3001)])
+def test_streamed_outputs_of_odd_rows(hip, rows, columns):
+    """Outputs past the last-level cache's size, on both layouts, with a partial
+    quad a row: sampled rows bit for bit, and nothing else written."""
+    banner(f"streamed outputs {rows}x{columns}")
+    assert 4 * rows * columns > 2 ** 28
+    g = torch.Generator("cuda").manual_seed(columns)
+    x = torch.randn(rows, columns, generator=g, device="cuda")
+    got = device.rows(hip.ROWS_SOFTMAX, x, hip.EXACT)
+    picked = torch.tensor(sorted({0, 1, 2, 3, rows // 2, rows - 2, rows - 1}), device="cuda")
+    assert_bitwise(got[picked], oracle.softmax_rows(x[picked].cpu().numpy()), f"softmax {rows}x{columns}")
+    ones = got.double().sum(1)
+    assert bool(((ones - 1).abs() < 1e-3).all())
