@@ -1225,12 +1225,13 @@ struct RowBlocking {
 
 // Points of four columns: rows of whole quads, and rows of eight or more
 // columns whose inputs are read along the row (unit or zero inner stride) or
-// by index, their last, partial quad lane by lane. One column a point costs
-// four times the loads, LDS accesses and stores: on MI355X, exact LayerNorm
-// over [8192, 2047] went from 164 to 85 us and over [4096, 50257] from 1297 to
-// 856 (one read 260 us), softmax over [6390, 3470] from 142 to 90, the
-// log-sum-exp over [4096, 50257] from 619 to 493; a lone row sum over
-// [6390, 3470] from 25.5 to 27.1.
+// by index. One column a point costs four times the loads, LDS accesses and
+// stores: on MI355X, exact LayerNorm over [8192, 2047] went from 161 to 77 us
+// and over [4096, 50257] from 1295 to 842 (one read 260 us), softmax over
+// [6390, 3470] from 142 to 91, the log-sum-exp over [4096, 50257] from 593 to
+// 442. Over 18 ragged shapes none is slower but for lone row sums and maxima a
+// few columns past a whole number of streamed slabs, by up to 5% (the maximum
+// over [33000, 2051] 53.7 and 56.2).
 bool row_quads(const RowProgram &p) {
   const int64_t c = p.columns();
   if (c % 4 == 0) return true;
@@ -1268,6 +1269,13 @@ RowBlocking row_blocking(const RowProgram &p) {
   while (b.rows > 8 && (rows + b.rows - 1) / b.rows < 1024) b.rows /= 2;
   const int per_lane = b.width == 4 ? 8 : 16;
   b.slab = per_lane * 256 * b.width / b.rows;
+  // Rows that are not whole quads and leave much of their last slab empty take
+  // slabs of half the width (on MI355X, with one column a point, whole and half
+  // slabs: the row sum over [9000, 2305] 21.5, 28.2 and 19.8 us, [6390, 3470]
+  // 26.4, 27.6 and 24.7, LayerNorm over the latter 137, 111 and 80; where the
+  // last slab is nearly full whole slabs are faster, softmax over [60000, 2999]
+  // 663, 644 and 736).
+  if (c % 4 != 0 && b.width == 4 && (c + b.slab - 1) / b.slab * b.slab * 20 >= c * 23) b.slab /= 2;
   return b;
 }
 
@@ -1411,12 +1419,40 @@ struct RowEmit {
     }
     s << indent << "}\n";
   }
-  // Stores full node k's four columns at `base`[at], the quad's first column
-  // being `col` of the row.
+  // Rows that are not whole quads. Resident: a row's last, partial point reads,
+  // computes and stores the row's last four columns, some of them as their own
+  // point does too (the same bits), and only parks shifted, so that no lane
+  // leaves its wave's path: most waves hold a partial point, and lane by lane
+  // loads and stores took up to a quarter of a row maximum or a LayerNorm
+  // ([200000, 65] 43 us, now 34; one column a point 34). `col` is the point's
+  // column, `back` the one it works from. Streamed rows, with few partial
+  // points, take theirs lane by lane.
+  bool overlaps() const { return p.columns() % 4 != 0; }
+  void emit_back(std::ostringstream &s, const std::string &back, const std::string &col, const std::string &indent) const {
+    s << indent << "const long long " << back << " = ";
+    if (overlaps())
+      s << "(" << col << ") > " << ll(p.columns() - 4) << " ? " << ll(p.columns() - 4) << " : (" << col << ");\n";
+    else
+      s << col << ";\n";
+  }
+  // Parks a point's four fold operands at their columns in LDS (the lanes past
+  // the row's end hold whatever; no fold reads them).
+  void park_quad(std::ostringstream &s, const std::string &slot, const std::string &list, const std::string &col,
+                 const std::string &indent) const {
+    if (!overlaps()) {
+      s << indent << "*(float4*)&" << slot << " = make_float4(" << list << ");\n";
+      return;
+    }
+    static const char *const shifted[4] = {"", "q.w, q.w, q.w, q.w", "q.z, q.w, q.w, q.w", "q.y, q.z, q.w, q.w"};
+    s << indent << "{ const float4 q = make_float4(" << list << "); *(float4*)&" << slot << " = (" << col << ") > "
+      << ll(p.columns() - 4) << " ? make_float4(" << shifted[p.columns() % 4] << ") : q; }\n";
+  }
+  // Stores full node k's four columns at `base`[at]; with `col`, a partial
+  // point lane by lane from that column on.
   void store_quad(std::ostringstream &s, const std::string &base, int k, const std::vector<std::string> &lanes,
-                  const std::string &col, const std::string &indent) const {
+                  const std::string &indent, const std::string &col = "") const {
     auto value = [&](int j) { return "f" + std::to_string(k) + "_" + lanes[j]; };
-    const bool partial = p.columns() % 4 != 0;
+    const bool partial = !col.empty() && overlaps();
     if (partial) s << indent << "if (" << col << " + 3 < " << ll(p.columns()) << ")\n  ";
     // An output of the last-level cache's size (256 MB) or more streams past
     // it: in a same-box A/B on MI355X the GPT-2 attention layer (402 MB of
@@ -1546,6 +1582,7 @@ Generated generate_row_resident(const RowProgram &p, const RowLayout &l, const R
       s << "  const bool ok" << I << " = q" << I << " < " << (int64_t)G * CV << " && row0 + r" << I << " < " << ll(R)
         << ";\n";
     }
+    if (V == 4) m.emit_back(s, "back" + I, "col" + I, "  ");
     const std::vector<std::string> lanes = lanes_of(i);
     for (size_t k = 0; k < p.inputs.size(); ++k) {
       if (!inputs_all[k]) continue;
@@ -1560,9 +1597,9 @@ Generated generate_row_resident(const RowProgram &p, const RowLayout &l, const R
     s << "    const long long g_r" << I << " = row0 + r" << I << ";\n";
     std::vector<std::string> c;
     if (p.rank > 1) emit_coordinates(s, p.rank - 1, p.shape, "g_r" + I, "r" + I, c);
-    c.push_back("col" + I);
+    c.push_back(V == 4 ? "back" + I : "col" + I);
     if (V == 4) {
-      m.load_quad(s, c, "r" + I, lanes, "    ", loaded, C % 4 != 0);
+      emit_quad_inputs(s, m.e, c, "r" + I, lanes, "    ", &loaded, false, true);
     } else {
       for (size_t k = 0; k < p.inputs.size(); ++k)
         if (loaded[k]) s << "    " << ref(-(int)k - 1, lanes[0]) << " = " << scalar_value(m.e, (int)k, c) << ";\n";
@@ -1586,7 +1623,7 @@ Generated generate_row_resident(const RowProgram &p, const RowLayout &l, const R
         m.emit_nodes(s, nodes_needed, lanes, "r" + I, "    ");
         if (V == 4) {
           const std::string list = m.fold_operands4(s, f, lanes, "r" + I, "    ", I);
-          s << "    *(float4*)&slab[r" << I << "][col" << I << "] = make_float4(" << list << ");\n";
+          m.park_quad(s, "slab[r" + I + "][col" + I + "]", list, "col" + I, "    ");
         } else {
           s << "    slab[r" << I << "][col" << I << "] = " << m.fold_operand(f, lanes[0], "r" + I) << ";\n";
         }
@@ -1641,14 +1678,15 @@ Generated generate_row_resident(const RowProgram &p, const RowLayout &l, const R
       if (p.transposed_outputs)
         s << "    const long long at = col" << I << " * " << ll(R) << " + row0 + r" << I << ";\n";
       else
-        s << "    const long long at = (row0 + r" << I << ") * " << ll(C) << " + col" << I << ";\n";
+        s << "    const long long at = (row0 + r" << I << ") * " << ll(C) << " + " << (V == 4 ? "back" : "col") << I
+          << ";\n";
       for (size_t o = 0; o < p.full_outputs.size(); ++o) {
         const int k = p.full_outputs[o];
         if (p.transposed_outputs)
           for (int j = 0; j < V; ++j)
             s << "    fo" << o << "[at + " << ll(j * R) << "] = f" << k << "_" << lanes[j] << ";\n";
         else if (V == 4)
-          m.store_quad(s, "fo" + std::to_string(o), k, lanes, "col" + I, "    ");
+          m.store_quad(s, "fo" + std::to_string(o), k, lanes, "    ");
         else
           s << "    fo" << o << "[at] = f" << k << "_" << lanes[0] << ";\n";
       }
@@ -1868,7 +1906,7 @@ Generated generate_row_streaming(const RowProgram &p, const RowLayout &l, const 
           for (int j = 0; j < V; ++j)
             s << "      fo" << o << "[at + " << ll(j * R) << "] = f" << k << "_" << lanes[j] << ";\n";
         else if (V == 4)
-          m.store_quad(s, "fo" + std::to_string(o), k, lanes, "(c0 + cu" + I + ")", "      ");
+          m.store_quad(s, "fo" + std::to_string(o), k, lanes, "      ", "(c0 + cu" + I + ")");
         else
           s << "      fo" << o << "[at] = f" << k << "_" << lanes[0] << ";\n";
       }
