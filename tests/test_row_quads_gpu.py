@@ -121,3 +121,23 @@ def test_streamed_outputs_of_odd_rows(hip, rows, columns):
     assert_bitwise(got[picked], oracle.softmax_rows(x[picked].cpu().numpy()), f"softmax {rows}x{columns}")
     ones = got.double().sum(1)
     assert bool(((ones - 1).abs() < 1e-3).all())
+
+
+@pytest.mark.parametrize("extent", [1, 3, 31, 32, 33, 383, 384, 385, 415, 416, 417, 767, 768, 769, 1151, 1155, 1537])
+@pytest.mark.parametrize("outputs", [16, 20, 100])
+def test_column_folds_at_their_tiles_edges(hip, extent, outputs):
+    """Ordered column sums around tiles of 384 steps, folded 32 at a time."""
+    from poorgrad_amd.topos import Tape
+
+    banner(f"column fold {extent}x{outputs}")
+    g = oracle.Generator(extent * 3 + outputs)
+    x, y = (g.normal(extent * outputs, 1.0).reshape(extent, outputs) for _ in range(2))
+    x[-1, 1], y[0, 2], x[0, 3] = np.inf, np.nan, -0.0
+    tape = Tape()
+    a, b = tape.input((extent, outputs)), tape.input((extent, outputs))
+    sums = [a.sum_along(0), (a * b + a).sum_along(0)]
+    feeds = {0: x, 1: y}
+    want = run_oracle(tape, sums, [], dense=feeds)
+    got, _ = run_device(tape, sums, [], dense=feeds, numerics=hip.EXACT)
+    for s in sums:
+        assert_bitwise(got[s.id], want[s.id], f"column fold {extent}x{outputs}")
