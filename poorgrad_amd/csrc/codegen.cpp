@@ -1466,14 +1466,16 @@ struct RowEmit {
     auto value = [&](int j) { return "f" + std::to_string(k) + "_" + lanes[j]; };
     const bool partial = !col.empty() && overlaps();
     if (partial) s << indent << "if (" << col << " + 3 < " << ll(p.columns()) << ")\n  ";
-    // An output of the last-level cache's size (256 MB) or more streams past
-    // it: in a same-box A/B on MI355X the GPT-2 attention layer (402 MB of
-    // weights and of their gradient) went from 2132 to 2103 us, and LayerNorm,
-    // softmax and a chain over [16384, 4096] from 500 to 478. (Chains keep
-    // plain stores: the 1.6 GB logits gradient streamed lost 0.6% of the
-    // two-layer GPT-2 step to the products that read it next.)
+    // An output well past the last-level cache's size (256 MB) streams past it.
+    // On MI355X, rows of 4096 written with plain stores and streamed, softmax
+    // over inputs not just read, 224 MB 175 and 182 us, 256 MB 194 and 204,
+    // 288 MB 247 and 253, 320 MB 283 and 276, 384 MB 314 and 302, 768 MB 644
+    // and 627; LayerNorm the same, and with a consumer of the output 2-5% more
+    // is won from 320 MB on and lost below. (Chains keep plain stores: the
+    // 1.6 GB logits gradient streamed lost 0.6% of the two-layer GPT-2 step to
+    // the products that read it next.)
     const std::string list = value(0) + ", " + value(1) + ", " + value(2) + ", " + value(3);
-    if (e.volume() * 4 >= (int64_t(1) << 28))
+    if (e.volume() * 4 >= (int64_t(5) << 26))
       s << indent << "__builtin_nontemporal_store(topos_f4{" << list << "}, (topos_f4*)(" << base << " + at));\n";
     else
       s << indent << "*(topos_f4*)(" << base << " + at) = topos_f4{" << list << "};\n";

@@ -108,12 +108,12 @@ def test_many_folds_over_streamed_rows(hip, rows, columns):
     assert_bitwise(got[total.id][rows_checked], want, f"many folds {rows}x{columns}")
 
 
-@pytest.mark.parametrize("rows, columns", [(1343, 50021), (262147, 257), (22370, 3001)])
+@pytest.mark.parametrize("rows, columns", [(1680, 50021), (330001, 257), (28001, 3001)])
 def test_streamed_outputs_of_odd_rows(hip, rows, columns):
     """Outputs past the last-level cache's size, on both layouts, with a partial
     quad a row: sampled rows bit for bit, and nothing else written."""
     banner(f"streamed outputs {rows}x{columns}")
-    assert 4 * rows * columns > 2 ** 28
+    assert 4 * rows * columns > 320 << 20
     g = torch.Generator("cuda").manual_seed(columns)
     x = torch.randn(rows, columns, generator=g, device="cuda")
     got = device.rows(hip.ROWS_SOFTMAX, x, hip.EXACT)
