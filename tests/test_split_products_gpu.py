@@ -233,6 +233,22 @@ def test_ranges_of_two_level_batches(hip, batch, heads, m, k, n):
     assert (np.abs(got[y.id] - merged(w, wide)) <= 1e-5 * merged(np.abs(w), np.abs(wide))).all()
 
 
+@pytest.mark.parametrize("left", [False, True])
+@pytest.mark.parametrize("right", [False, True])
+@pytest.mark.parametrize("m, k, n", [(2048, 16, 2048), (2048, 40, 2048), (4096, 64, 1024), (12544, 16, 72),
+                                     (8192, 512, 4096), (512, 16, 512)])
+def test_errors_do_not_add_up_over_rows_or_columns(hip, m, k, n, left, right):
+    """Independent errors of the size the product has average out: the mean
+    error of a row or a column lies within six standard deviations of zero."""
+    banner(f"mean errors {m}x{k}x{n} {left} {right}")
+    a, b = operand(61, m, k, left), operand(62, k, n, right)
+    error = product(hip, a, b).double() - a.double() @ b.double()
+    deviation = float(error.std())
+    for axis, count in ((0, m), (1, n)):
+        assert float(error.mean(axis).abs().max()) <= 6 * deviation / count ** 0.5
+    assert abs(float(error.mean())) <= 6 * deviation / (m * n) ** 0.5
+
+
 def test_zeros_are_positive(hip):
     """A product of zeros, signed or not, is +0."""
     banner("zeros")
